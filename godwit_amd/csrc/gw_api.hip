@@ -1379,7 +1379,7 @@ static int moe_prefill_impl(gw_expert_runner *r, const gw_moe_layer_args *a, int
         g.fdim = (int)(2 * r->inter);
         g.act_out = ps.act;
         g.y_out = nullptr;
-        ProfScope p(ctx, "prefill_gate_up");
+        ProfScope p(ctx, wide ? "prefill_gate_up_wide" : "prefill_gate_up");
         GW_HIP(gw::launch_prefill_gemm(p.launch(L), true, planes, g, max_tiles, hint));
     }
     {
@@ -1417,7 +1417,7 @@ static int moe_prefill_impl(gw_expert_runner *r, const gw_moe_layer_args *a, int
             g.comb_topk = K;
             g.comb_residual = out_mode == 2 ? 1 : 0;
         }
-        ProfScope p(ctx, "prefill_down");
+        ProfScope p(ctx, wide ? "prefill_down_wide" : "prefill_down");
         GW_HIP(gw::launch_prefill_gemm(p.launch(L), false, 1, g, max_tiles, hint));
     }
     if (!fuse_combine) {

@@ -86,7 +86,9 @@ int gw_context_cu_count(gw_context *ctx, int *cus);
  * while enabled, every launch is bracketed by hipEvents on the context stream.
  * gw_context_profile_read synchronises and returns the summed GPU milliseconds
  * and launch count of the kernel family `name` ("gate_up", "down", "route",
- * "router", "gemv", "dequant", "activation", "accumulate"). */
+ * "router", "gemv", "dequant", "activation", "accumulate"; of a batch
+ * "prefill_gate_up", "prefill_down", with "_wide" behind them for tiles of 96
+ * entries, "prefill_combine", "prefill_route", "prefill_group"). */
 int gw_context_set_profiling(gw_context *ctx, int enabled);
 int gw_context_profile_read(gw_context *ctx, const char *name, double *total_ms,
                             int64_t *launches);
@@ -270,8 +272,8 @@ int gw_expert_apply_assignments_async(gw_expert_runner *runner, const void *inpu
  * a kernel of its own; results are the same bytes either way.  Batches of many
  * entries per expert (24 per expert and 1152 in all; GODWIT_WIDE_ENTRIES at
  * runner creation sets a number per expert) use tiles of 96 entries instead of
- * 32: the same exact products, their fp32 sums in another order.  Enqueue
- * only. */
+ * 32: the same sums in the same order, so the same bytes while the scale bytes
+ * lie in [104, 140].  Enqueue only. */
 typedef struct gw_moe_layer_args {
     const uint8_t *experts_base;
     int64_t expert_stride;

@@ -16,7 +16,8 @@ import pytest
 import godwit_amd as gw
 import oracle
 from godwit_amd._lib import check, lib
-from helpers import ExpertData, expert_metric, layer_check, normal_bf16, rng
+from helpers import (ExpertData, expert_from_blob, expert_metric, fill_layer_device, layer_check,
+                     normal_bf16, rng)
 from test_gpu_expert import GPTOSS, QWEN3, SMALL, _make_layer
 
 pytestmark = pytest.mark.gpu
@@ -658,3 +659,78 @@ def test_wide_tiles_edge_scales(ctx, monkeypatch):
     test_prefill_edge_scales(ctx, 40)
     test_prefill_down_fp16_range(ctx, monkeypatch, 40, "")
     test_prefill_gate_up_fp16_x(ctx, monkeypatch, 40, "")
+
+
+def _fp64_layer(layout, blobs, ids, x, H, F, act):
+    """Top-1 outputs of every token in fp64 on the host, the activation rounded to fp16,
+    and how far each may be off: a last bit of a gate_up sum can round an activation one
+    fp16 step (2^-10 of it, 2^-24 at the least) the other way, and the fp32 sums of the
+    down projection are within 2^-16 of the sum of the terms' sizes."""
+    nb, fb, y = H // 32, F // 32, np.zeros((len(ids), H))
+    off = np.zeros((len(ids), H))
+    for e, blob in enumerate(blobs):
+        t = np.nonzero(ids == e)[0]
+        o = expert_from_blob(blob, layout).arrays
+        w = oracle.decode(o[0], o[1], 2 * F * nb).reshape(2 * F, H).astype(np.float64)
+        v = x[t].astype(np.float64) @ w.T + o[4].astype(np.float64)
+        g, u = v[:, 0::2], v[:, 1::2]
+        if act == "silu":
+            a = g / (1.0 + np.exp(-g)) * u
+        else:
+            g, u = np.minimum(g, 7.0), np.clip(u, -7.0, 7.0)
+            a = g / (1.0 + np.exp(-1.702 * g)) * (u + 1.0)
+        w = oracle.decode(o[2], o[3], H * fb).reshape(H, F).astype(np.float64)
+        y[t] = a.astype(np.float16).astype(np.float64) @ w.T + o[5].astype(np.float64)
+        off[t] = (np.abs(a) * (2.0 ** -10 + 2.0 ** -16) + 2.0 ** -24) @ np.abs(w).T
+    return y, off
+
+
+@pytest.mark.parametrize("x_dtype", [gw.BF16, gw.F16], ids=["bf16", "f16"])
+@pytest.mark.parametrize("H,F,act,E,entries", [
+    (2880, 2880, "gptOssClampedGLU", 6, "0"),   # 23 chunks, the last of two blocks
+    (2048, 768, "silu", 6, None),               # 16 and 6 chunks; the default rule
+    (352, 224, "silu", 6, "0"),                 # 3 and 2 chunks, 256 of K reached once
+], ids=["gptoss", "qwen3-default", "352x224"])
+def test_wide_tiles_same_bytes(ctx, monkeypatch, H, F, act, E, entries, x_dtype):
+    """The wide tiles' sums are those of the 32-entry tiles, MFMA step for MFMA step, so a
+    batch's outputs and activations are the same bytes (GODWIT_WIDE_ENTRIES keeps the other
+    runner on 32-entry tiles), at widths that go round the rings many times, in tiles of one,
+    two and three column groups; and they agree with fp64."""
+    counts = [20, 64, 65, 96, 130, 33] if entries else [1000, 30, 60, 97, 64, 1650]
+    T = sum(counts)
+    layout = gw.ExpertLayout(H, F, E)
+    r = rng(3800 + H)
+    buf = ctx.empty(layout.layer_file_size)
+    fill_layer_device(ctx, buf, layout, E, 3801)
+    for sec in ("gate_up_scales", "down_scales"):
+        ctx.fill_uniform_u8(buf, 117, 122, 3802, offset=layout.offsets[sec],
+                            count=layout.sizes[sec], rows=E, row_stride=layout.stride)
+    xb, xw = _x(ctx, r, T, H, x_dtype)
+    logits = np.zeros((T, E), np.float32)
+    logits[np.arange(T), r.permutation(np.repeat(np.arange(E), counts))] = 4.0
+    lb = ctx.buffer(logits)
+    got = {}
+    for tiles, env in (("wide", entries), ("32", "1000000")):
+        monkeypatch.delenv("GODWIT_WIDE_ENTRIES", raising=False)
+        if env:
+            monkeypatch.setenv("GODWIT_WIDE_ENTRIES", env)
+        runner = gw.ExpertRunner(ctx, H, F, act)
+        ctx.set_profiling(True)
+        ctx.profile_reset()
+        out, _, ids, _ = _run(ctx, runner, layout, buf, E, 1, xb, x_dtype, lb, T, H)
+        n = [ctx.profile(k)[1] for k in ("prefill_gate_up_wide", "prefill_down_wide",
+                                         "prefill_gate_up", "prefill_down")]
+        ctx.set_profiling(False)
+        assert n == ([1, 1, 0, 0] if tiles == "wide" else [0, 0, 1, 1]), (tiles, n)
+        act_bits = _download(ctx, runner.prefill_view()["activations"], np.uint16, T * F)
+        got[tiles] = out, act_bits, ids
+        runner.close()
+    for i in range(3):
+        assert np.array_equal(got["wide"][i], got["32"][i]), i
+    raw = buf.download(np.uint8, layout.stride * E).reshape(E, layout.stride)
+    y, off = _fp64_layer(layout, raw, got["wide"][2][:, 0], xw.reshape(T, H), H, F, act)
+    err = np.abs(got["wide"][0] - y)
+    assert np.all(err <= off), (err / off).max()
+    assert np.median(err.max(1) / np.abs(y).mean(1)) < 1e-4
+    for b in (xb, lb, buf):
+        b.free()
