@@ -1330,11 +1330,12 @@ static int moe_prefill_impl(gw_expert_runner *r, const gw_moe_layer_args *a, int
     // 49 -> 63 us against an 8.3 us combine), except when the down GEMM runs
     // the 4-wave shape, where it costs less (GPT-OSS 512 tokens: down 191 ->
     // 195 us against a 9 us combine and its launch gap).  The wide GEMM keeps
-    // it apart (GPT-OSS 4096 tokens: 492 us fused, 400 + 66 apart; Qwen3 1021
-    // tokens: 124 fused, 56 + 20 apart).
+    // it apart whatever the bound (GPT-OSS 4096 tokens: 492 us fused, 400 + 66
+    // apart; Qwen3 1021 tokens: 124 fused, 56 + 20 apart).
     const bool fuse_combine =
+        !wide &&
         (T <= r->fused_combine_max ||
-         (r->fused_combine_max > 0 && !wide &&
+         (r->fused_combine_max > 0 &&
           gw::prefill_down_four_wave((int)r->hidden, (int)r->inter, hint, max_tiles, L.cus))) &&
         (int64_t)sizeof(float) * T * K * r->hidden < ((int64_t)1 << 31);
     gw::PrefillGemm g;

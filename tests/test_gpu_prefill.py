@@ -734,3 +734,54 @@ def test_wide_tiles_same_bytes(ctx, monkeypatch, H, F, act, E, entries, x_dtype)
     assert np.median(err.max(1) / np.abs(y).mean(1)) < 1e-4
     for b in (xb, lb, buf):
         b.free()
+
+
+@pytest.mark.parametrize("T,E,entries,bound", [
+    (13, 16, "0", None), (17, 16, "0", None), (32, 16, "0", None), (2048, 8, None, "100000"),
+    (300, 8, "0", "0")])
+def test_wide_tiles_any_combine_bound(ctx, monkeypatch, T, E, entries, bound):
+    """Wide tiles never combine in their down GEMM: batches below the fused-combine bound that
+    GODWIT_WIDE_ENTRIES sends to them (13 tokens are the first past self-grouping), and
+    batches of the default rule under a raised GODWIT_FUSED_COMBINE_TOKENS, run and give the
+    bytes of the 32-entry tiles, eagerly and replayed."""
+    shape, K = SMALL, 8
+    H, F = shape["hidden"], shape["inter"]
+    layout, experts, buf = _make_layer(ctx, shape, E, 3900)
+    r = rng(3901 + T)
+    xb, _ = _x(ctx, r, T, H, gw.BF16)
+    logits = r.standard_normal((T, E)).astype(np.float32)
+    lb = ctx.buffer(logits)
+    runs = {}
+    for tiles in ("32", "wide"):
+        for name, value in (("GODWIT_WIDE_ENTRIES", entries if tiles == "wide" else "1000000"),
+                            ("GODWIT_FUSED_COMBINE_TOKENS", bound if tiles == "wide" else None)):
+            monkeypatch.delenv(name, raising=False)
+            if value is not None:
+                monkeypatch.setenv(name, value)
+        runner = gw.ExpertRunner(ctx, H, F, shape["act"])
+        ctx.set_profiling(True)
+        ctx.profile_reset()
+        runs[tiles] = _run(ctx, runner, layout, buf, E, K, xb, gw.BF16, lb, T, H)
+        n = ctx.profile("prefill_down_wide")[1], ctx.profile("prefill_combine")[1]
+        ctx.set_profiling(False)
+        if tiles == "wide":
+            assert n == (1, 1), n
+            out = ctx.empty(T * H * 4)
+
+            def body():
+                runner.prefill_forward(buf.ptr, layout.stride, E, K, xb.ptr, gw.BF16, T, out.ptr,
+                                       logits=lb.ptr)
+
+            graph = gw.Graph.capture(ctx, body)
+            for _ in range(3):
+                out.zero()
+                graph.launch()
+                ctx.synchronize()
+                assert np.array_equal(out.download(np.float32, T * H), runs["32"][0].ravel())
+            graph.destroy()
+            out.free()
+        runner.close()
+    for i in range(4):
+        assert np.array_equal(runs["wide"][i], runs["32"][i]), i
+    for b in (xb, lb, buf):
+        b.free()
