@@ -18,6 +18,7 @@ package fails when the library has not been built.
 from __future__ import annotations
 
 import ctypes
+import operator
 import os
 import struct
 from dataclasses import dataclass, field
@@ -44,6 +45,7 @@ SECTIONS = ["gate_up_blocks", "gate_up_scales", "down_blocks", "down_scales",
 ACTIVATIONS = {"gptOssClampedGLU": ACT_GPTOSS_CLAMPED_GLU, "silu": ACT_SILU}
 
 _ASSIGNMENT = struct.Struct("=Q6qif")          # AssignmentC
+_SECTION_OFFSETS = operator.itemgetter(*SECTIONS)
 assert _ASSIGNMENT.size == ctypes.sizeof(AssignmentC)
 
 _NP_DTYPES = {F32: np.float32, F16: np.float16, BF16: np.uint16}
@@ -422,21 +424,23 @@ class ExpertRunner:
         n = len(assignments)
         if n == 0:
             return
-        # AssignmentC records packed in one buffer; a list's weights mostly share one
-        # offsets dict, read once per call.
+        # AssignmentC records packed in one buffer.  Every element is read as it comes,
+        # its offsets too: a sequence may make its elements, or change a dict, as it goes.
         arr = (AssignmentC * n)()
-        size, pack, seen = _ASSIGNMENT.size, _ASSIGNMENT.pack_into, {}
+        size, pack, at = _ASSIGNMENT.size, _ASSIGNMENT.pack_into, _SECTION_OFFSETS
         for i, a in enumerate(assignments):
             w = a.weights
-            offs = seen.get(id(w.offsets))
-            if offs is None:
-                offs = seen[id(w.offsets)] = [int(w.offsets.get(s, 0)) for s in SECTIONS]
-            try:
-                pack(arr, i * size, w.address(), *offs, int(a.token), float(a.routing_weight))
-            except (struct.error, OverflowError):    # a value that ctypes wraps or rounds
-                arr[i].weights = w.c()
-                arr[i].token = int(a.token)
-                arr[i].routing_weight = float(a.routing_weight)
+            if type(w) is Weights and type(w.offsets) is dict:
+                b = w.buffer
+                try:
+                    pack(arr, i * size, b if type(b) is int else w.address(), *at(w.offsets),
+                         int(a.token), a.routing_weight)
+                    continue
+                except (KeyError, struct.error, OverflowError):
+                    pass          # a section left out, or a value that ctypes converts
+            arr[i].weights = w.c()
+            arr[i].token = int(a.token)
+            arr[i].routing_weight = float(a.routing_weight)
         fn = lib.gw_expert_apply_assignments if wait else lib.gw_expert_apply_assignments_async
         check(fn(self.handle, inputs.ptr, dtype, arr, n, outputs.ptr))
 

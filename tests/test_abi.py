@@ -107,3 +107,73 @@ def test_errors_without_device():
     w = np.zeros(8, np.float32)
     assert _lib.lib.gw_router_select(lg.ctypes.data, 4, 5, ids.ctypes.data,
                                      w.ctypes.data) == _lib.GW_ERR_SHAPE
+
+
+def test_assignment_records_are_read_element_by_element(monkeypatch):
+    """apply_assignments hands the library one record an element, each with that element's
+    own offsets: for a list, for a sequence that makes its elements as it is read (a dict
+    freed before the next one is made may leave it its place), for one dict changed between
+    elements, and for values that the packed form does not take (a section left out, a dict
+    subclass, a float offset, a weight past fp32's range)."""
+    import godwit_amd as gw
+    from godwit_amd._lib import AssignmentC
+    seen = []
+
+    def record(handle, x, dtype, arr, n, out):
+        size = ctypes.sizeof(AssignmentC)
+        raw = ctypes.string_at(ctypes.addressof(arr), n * size)
+        seen.append([AssignmentC.from_buffer_copy(raw, i * size) for i in range(n)])
+        return 0
+
+    class Lib:
+        gw_expert_apply_assignments = staticmethod(record)
+
+    monkeypatch.setattr(gw, "lib", Lib)
+    runner = gw.ExpertRunner.__new__(gw.ExpertRunner)
+    runner.handle = None
+
+    class Buf:
+        ptr = 0
+
+    def offsets(i):
+        return {s: 1000 * i + k for k, s in enumerate(gw.SECTIONS)}
+
+    def element(i):
+        return gw.Assignment(gw.Weights(4096 + i, offsets(i)), i % 3, 0.25 * i)
+
+    class Lazy:
+        def __len__(self):
+            return 24
+
+        def __iter__(self):
+            return (element(i) for i in range(24))
+
+    shared = {}
+
+    def changed():
+        for i in range(24):
+            shared.update(offsets(i))
+            yield gw.Assignment(gw.Weights(4096 + i, shared), i % 3, 0.25 * i)
+
+    class Changed(Lazy):
+        def __iter__(self):
+            return changed()
+
+    class Sub(dict):
+        def __missing__(self, key):
+            raise AssertionError("an absent section is offset 0")
+
+    for seq in ([element(i) for i in range(24)], Lazy(), Changed()):
+        runner.apply_assignments(Buf, seq, Buf)
+        for i, r in enumerate(seen.pop()):
+            assert list(r.weights.offsets) == list(offsets(i).values()), i
+            assert (r.weights.buffer, r.token, r.routing_weight) == (4096 + i, i % 3, 0.25 * i)
+    less = {gw.SECTIONS[1]: 7}
+    runner.apply_assignments(Buf, [
+        gw.Assignment(gw.Weights(1, less), 0, 1.0), gw.Assignment(gw.Weights(1, Sub(less)), 0, 1.0),
+        gw.Assignment(gw.Weights(1, {**offsets(2), gw.SECTIONS[0]: 5.0}), 0, 1e39)], Buf)
+    a, b, c = seen.pop()
+    assert list(a.weights.offsets) == list(b.weights.offsets) == [0, 7, 0, 0, 0, 0]
+    assert list(c.weights.offsets) == [5] + list(offsets(2).values())[1:]
+    assert c.routing_weight == float("inf")
+    assert len(less) == 1
