@@ -804,7 +804,8 @@ __global__ __launch_bounds__(256) void router_rows_kernel(const void *__restrict
 // workgroup (32 tokens, 32 experts), its 16 waves a sixteenth of K each, whose
 // partial tiles meet in LDS and are added in wave order plus the bias.  The
 // products are exact (an fp16 x enters as hi + lo, two bf16 values whose sum it
-// is), a wave's sum is a few MFMA steps long.  router_rows_kernel reads a
+// is; infinities and NaN give what one product would), a wave's sum is a few
+// MFMA steps long.  router_rows_kernel reads a
 // weight row for each 8 tokens with one product a lane-op.  us a launch, rows /
 // matrix cores: Qwen3 (128 experts) 128 tokens 17 / 10, 1021 107 / 12, 4096 421
 // / 27; GPT-OSS 128 experts 64 tokens 12 / 20, 128 17 / 18, 512 61 / 17; 32
@@ -831,41 +832,63 @@ __global__ __launch_bounds__(1024) void router_mfma_kernel(const uint16_t *__res
     const int steps = H >> 4;
     const int s0 = wave * steps / kWaves, s1 = (wave + 1) * steps / kWaves;
     f32x16 acc;
+    // NONFINITE: an infinite x is its hi alone (v - hi would be NaN), and an
+    // infinite or NaN weight meets no lo (which is 0 where x is its hi).
+    auto add_up = [&](auto nonfinite) {
+        constexpr bool NONFINITE = decltype(nonfinite)::value;
 #pragma unroll
-    for (int v = 0; v < 16; ++v) acc[v] = 0.0f;
-    for (int s = s0; s < s1; s += kU) {
-        uint4 a[kU], v[kU];
+        for (int v = 0; v < 16; ++v) acc[v] = 0.0f;
+        for (int s = s0; s < s1; s += kU) {
+            uint4 a[kU], v[kU];
 #pragma unroll
-        for (int u = 0; u < kU; ++u) {
-            const int at = 16 * min(s + u, s1 - 1);
-            a[u] = *reinterpret_cast<const uint4 *>(wr + at);
-            v[u] = *reinterpret_cast<const uint4 *>(xr + at);
-        }
+            for (int u = 0; u < kU; ++u) {
+                const int at = 16 * min(s + u, s1 - 1);
+                a[u] = *reinterpret_cast<const uint4 *>(wr + at);
+                v[u] = *reinterpret_cast<const uint4 *>(xr + at);
+            }
 #pragma unroll
-        for (int u = 0; u < kU; ++u) {
-            if (s + u >= s1) break;                   // uniform
-            const bf16x8 aw = __builtin_bit_cast(bf16x8, a[u]);
-            if constexpr (XDT == DT_BF16) {
-                acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(aw, __builtin_bit_cast(bf16x8, v[u]), acc, 0, 0, 0);
-            } else {
-                const uint32_t r[4] = {v[u].x, v[u].y, v[u].z, v[u].w};
-                uint32_t hi[4], lo[4];
+            for (int u = 0; u < kU; ++u) {
+                if (s + u >= s1) break;               // uniform
+                const bf16x8 aw = __builtin_bit_cast(bf16x8, a[u]);
+                if constexpr (XDT == DT_BF16) {
+                    acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(aw, __builtin_bit_cast(bf16x8, v[u]), acc, 0, 0, 0);
+                } else {
+                    const uint32_t r[4] = {v[u].x, v[u].y, v[u].z, v[u].w};
+                    uint32_t wl[4] = {a[u].x, a[u].y, a[u].z, a[u].w};
+                    uint32_t hi[4], lo[4];
 #pragma unroll
-                for (int k = 0; k < 4; ++k) {
-                    const float v0 = f16_bits_to_f32((uint16_t)r[k]);
-                    const float v1 = f16_bits_to_f32((uint16_t)(r[k] >> 16));
-                    const uint32_t b0 = __float_as_uint(v0) & 0xFFFF0000u;
-                    const uint32_t b1 = __float_as_uint(v1) & 0xFFFF0000u;
-                    hi[k] = (b0 >> 16) | b1;
-                    lo[k] = (__float_as_uint(v0 - __uint_as_float(b0)) >> 16) |
-                            (__float_as_uint(v1 - __uint_as_float(b1)) & 0xFFFF0000u);
+                    for (int k = 0; k < 4; ++k) {
+                        const float v0 = f16_bits_to_f32((uint16_t)r[k]);
+                        const float v1 = f16_bits_to_f32((uint16_t)(r[k] >> 16));
+                        const uint32_t b0 = __float_as_uint(v0) & 0xFFFF0000u;
+                        const uint32_t b1 = __float_as_uint(v1) & 0xFFFF0000u;
+                        hi[k] = (b0 >> 16) | b1;
+                        lo[k] = (__float_as_uint(v0 - __uint_as_float(b0)) >> 16) |
+                                (__float_as_uint(v1 - __uint_as_float(b1)) & 0xFFFF0000u);
+                        if constexpr (NONFINITE) {
+                            if ((r[k] & 0x7FFFu) == 0x7C00u) lo[k] &= 0xFFFF0000u;
+                            if ((r[k] & 0x7FFF0000u) == 0x7C000000u) lo[k] &= 0x0000FFFFu;
+                            if ((wl[k] & 0x7F80u) == 0x7F80u) wl[k] &= 0xFFFF0000u;
+                            if ((wl[k] & 0x7F800000u) == 0x7F800000u) wl[k] &= 0x0000FFFFu;
+                        }
+                    }
+                    acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
+                        __builtin_bit_cast(bf16x8, make_uint4(wl[0], wl[1], wl[2], wl[3])),
+                        __builtin_bit_cast(bf16x8, make_uint4(lo[0], lo[1], lo[2], lo[3])), acc, 0, 0, 0);
+                    acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
+                        aw, __builtin_bit_cast(bf16x8, make_uint4(hi[0], hi[1], hi[2], hi[3])), acc, 0, 0, 0);
                 }
-                acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
-                    aw, __builtin_bit_cast(bf16x8, make_uint4(lo[0], lo[1], lo[2], lo[3])), acc, 0, 0, 0);
-                acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
-                    aw, __builtin_bit_cast(bf16x8, make_uint4(hi[0], hi[1], hi[2], hi[3])), acc, 0, 0, 0);
             }
         }
+    };
+    add_up(std::false_type{});
+    if constexpr (XDT == DT_F16) {
+        // An infinity or NaN among the inputs always shows in a sum: only then
+        // is the share summed once more (a check of every step took 4 us).
+        bool finite = true;
+#pragma unroll
+        for (int v = 0; v < 16; ++v) finite &= fabsf(acc[v]) < __builtin_inff();
+        if (__ballot(!finite)) add_up(std::true_type{});
     }
 #pragma unroll
     for (int v = 0; v < 16; ++v) {

@@ -373,3 +373,47 @@ def test_router_logits_batch(ctx, experts, hidden, tokens, x_dtype, bias):
     assert np.all(np.abs(got - want) <= size * 2.0 ** -20)
     for b in (wbuf, xbuf, out) + ((bb,) if bb else ()):
         b.free()
+
+
+@pytest.mark.parametrize("x_dtype", [gw.F16, gw.BF16], ids=["f16", "bf16"])
+def test_router_logits_batch_non_finite(ctx, x_dtype):
+    """Infinities and NaN in x and in the weights, in a batch on the matrix cores and in the
+    same rows taken 8 at a time (below 16384 logits): both give the infinities and NaN of the
+    exact sums (inf * 0 and inf - inf are NaN), and finite logits elsewhere."""
+    experts, hidden, tokens = 64, 96, 256
+    r = rng(7800)
+    w = (0.05 * r.standard_normal((experts, hidden))).astype(np.float32)
+    x = r.standard_normal((tokens, hidden)).astype(np.float32)
+    x[:, 3] = 0.5                       # exact in 8 bits: no lo
+    x[40:44, 3] = 0.0
+    w[5, 3], w[6, 3], w[7, 9], w[8, 3:5] = np.inf, -np.inf, np.nan, (np.inf, -np.inf)
+    w[9:12, 70], w[13, :] = 0.0, np.inf
+    x[17, 70], x[18, 71], x[19, 70:72], x[20, 5] = np.inf, -np.inf, (np.inf, -np.inf), np.nan
+    x[33, :] = -np.inf
+    wb = oracle.f32_to_bf16_bits(w.ravel())
+    w = oracle.bf16_bits_to_f32(wb).astype(np.float64).reshape(experts, hidden)
+    if x_dtype == gw.F16:
+        xb = x.astype(np.float16)
+        x = xb.astype(np.float64)
+    else:
+        xb = oracle.f32_to_bf16_bits(x.ravel())
+        x = oracle.bf16_bits_to_f32(xb).astype(np.float64).reshape(tokens, hidden)
+    wbuf, xbuf, out = ctx.buffer(wb), ctx.buffer(xb), ctx.empty(tokens * experts * 4)
+
+    def logits(t0, n):
+        check(lib.gw_router_logits(ctx.handle, wbuf.ptr, gw.BF16, None, gw.BF16,
+                                   xbuf.ptr + t0 * hidden * 2, x_dtype, out.ptr, experts, hidden, n))
+        return out.download(np.float32, n * experts).reshape(n, experts)
+
+    batch = logits(0, tokens)
+    rows = np.concatenate([logits(t, 8) for t in range(0, tokens, 8)])
+    with np.errstate(invalid="ignore"):
+        terms = x[:, None, :] * w[None, :, :]
+        want, size = terms.sum(2), np.abs(terms).sum(2)
+    finite = np.isfinite(want)
+    assert np.isnan(want).any() and np.isposinf(want).any() and np.isneginf(want).any()
+    for got in (batch, rows):
+        assert np.array_equal(np.where(finite, 0.0, got), np.where(finite, 0.0, want), equal_nan=True)
+        assert np.all(np.abs(got[finite] - want[finite]) <= size[finite] * 2.0 ** -20)
+    for b in (wbuf, xbuf, out):
+        b.free()
