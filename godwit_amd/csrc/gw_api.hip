@@ -1300,14 +1300,24 @@ static int moe_prefill_impl(gw_expert_runner *r, const gw_moe_layer_args *a, int
     // has a part that grows with the experts and a fixed one (a quarter of the
     // workgroups, so a last round of them costs more), and is less than that
     // of the 32-entry tiles from 24 entries an expert and 1152 in all.  us a
-    // layer, 32-entry tiles / wide: GPT-OSS 128 experts, 3072 entries 601 /
-    // 591, 4096 669 / 632, 8192 938 / 777, 16384 1582 / 1165; 32 experts, 1280
-    // 195 / 211, 1536 217 / 223, 2048 251 / 234, 4096 433 / 338; Qwen3, 4096
-    // 153 / 158, 6144 192 / 181, 8192 222 / 196, 16384 388 / 296.
+    // layer, 32-entry tiles / wide, uniform routing: GPT-OSS, 128 experts, 3584
+    // entries 513 / 588, 4352 616 / 613, 5120 707 / 626, 8192 882 / 702, 12288
+    // 1204 / 968 (Zipf(1.1): 4608 657 / 681, 5632 739 / 729, 12288 1230 / 990);
+    // 64 experts, 2304 340 / 345, 2816 368 / 351, 4096 462 / 391; 32 experts,
+    // 1024 163 / 206, 1792 209 / 211, 2048 235 / 235, 2560 281 / 229; Qwen3,
+    // 128 experts, 4096 145 / 148, 4608 167 / 155, 8192 229 / 181; 4096 x 1536,
+    // 128 experts, 3072 382 / 387, 4096 471 / 418.  (16 GPT-OSS experts lose
+    // at 1536, 156 / 188, where their tiles are half full, and gain from 2048,
+    // 202 / 183.)
+    // Narrow layers want more: below 16384 / (256-row tiles of gate_up) entries
+    // the full tiles are fewer than two thirds of the CUs.  2048 x 768, 8 / 16
+    // experts, 1536 entries 60 / 68 and 61 / 69, 2048 71 / 69 and 71 / 71, 3072
+    // (16) 89 / 80; 1024 x 512, 32 experts, 2048 45 / 52, 3072 53 / 57, 4096 67 / 58.
+    const int64_t entries = (int64_t)T * K, ftiles = (2 * r->inter + 255) / 256;
+    const bool many = r->wide_entries >= 0 ? entries >= (int64_t)r->wide_entries * E
+                                           : entries >= (int64_t)24 * E + 1152 && entries * ftiles >= 16384;
     const bool wide = !self_group && gw::prefill_planes(a->x_dtype) == 1 && r->gemm_waves == 0 &&
-                      (int64_t)T * K >= (r->wide_entries >= 0 ? (int64_t)r->wide_entries * E
-                                                              : (int64_t)24 * E + 1152) &&
-                      r->hidden * r->inter < ((int64_t)1 << 31);   // 32-bit buffer offsets
+                      many && r->hidden * r->inter < ((int64_t)1 << 31);   // 32-bit buffer offsets
     const int tile = wide ? gw::kWideTile : 32;
     const int hint = gw::prefill_tiles_hint(T, K, E);
     const int max_tiles = self_group ? std::min(E, T * K) : gw::prefill_max_tiles(T, K, E, tile);

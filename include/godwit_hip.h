@@ -270,10 +270,11 @@ int gw_expert_apply_assignments_async(gw_expert_runner *runner, const void *inpu
  * group kernel's tile list.  Up to GODWIT_FUSED_COMBINE_TOKENS tokens (default
  * 32, 0 disables) the weighted combine runs inside the down GEMM instead of
  * a kernel of its own; results are the same bytes either way.  Batches of many
- * entries per expert (24 per expert and 1152 in all; GODWIT_WIDE_ENTRIES at
- * runner creation sets a number per expert) use tiles of 96 entries instead of
- * 32: the same sums in the same order, so the same bytes while the scale bytes
- * lie in [104, 140].  Enqueue only. */
+ * entries per expert (24 per expert and 1152 in all, and at least 16384 /
+ * ceil(gate_up rows / 256); GODWIT_WIDE_ENTRIES at runner creation sets a number
+ * per expert instead) use tiles of 96 entries instead of 32: the same sums in
+ * the same order, so the same bytes while the scale bytes lie in [104, 140].
+ * Enqueue only. */
 typedef struct gw_moe_layer_args {
     const uint8_t *experts_base;
     int64_t expert_stride;

@@ -785,3 +785,32 @@ def test_wide_tiles_any_combine_bound(ctx, monkeypatch, T, E, entries, bound):
         assert np.array_equal(runs["wide"][i], runs["32"][i]), i
     for b in (xb, lb, buf):
         b.free()
+
+
+@pytest.mark.parametrize("shape,E,K,T", [
+    (SMALL, 8, 8, 2048),                            # one 256-row tile: 16384 entries
+    (dict(SMALL, inter=1792), 8, 8, 168),           # 14 of them: 24 an expert and 1152
+])
+def test_wide_tiles_default_rule(ctx, shape, E, K, T):
+    """The wide tiles start where the rule says: the batch at the line takes them, one token
+    less does not, and nor does an fp32 x."""
+    H, F = shape["hidden"], shape["inter"]
+    layout = gw.ExpertLayout(H, F, E)
+    buf = ctx.empty(layout.layer_file_size)
+    fill_layer_device(ctx, buf, layout, E, 4001)
+    runner = gw.ExpertRunner(ctx, H, F, shape["act"])
+    r = rng(4000 + T)
+    lb = ctx.buffer(r.standard_normal((T, E)).astype(np.float32))
+    for x_dtype, tokens, wide in ((gw.BF16, T, 1), (gw.F16, T, 1), (gw.BF16, T - 1, 0),
+                                  (gw.F16, T - 1, 0), (gw.F32, T, 0)):
+        xb, _ = _x(ctx, r, tokens, H, x_dtype)
+        ctx.set_profiling(True)
+        ctx.profile_reset()
+        _run(ctx, runner, layout, buf, E, K, xb, x_dtype, lb, tokens, H)
+        n = ctx.profile("prefill_gate_up_wide")[1], ctx.profile("prefill_gate_up")[1]
+        ctx.set_profiling(False)
+        assert n == (wide, 1 - wide), (x_dtype, tokens, n)
+        xb.free()
+    for b in (lb, buf):
+        b.free()
+    runner.close()
