@@ -1079,7 +1079,12 @@ int prefill_gemm_lds_bytes(int planes, int kdim, int waves, int depth)
 // spread by 128 rows instead of 256 (us, the other shapes / this; GPT-OSS 2
 // tokens down 26 / 20, 6 tokens down 46 / 35, 4 tokens gate_up 42 / 40, fp16
 // 47 / 40, 16 fp16 tokens of 32 experts down 47 / 38; Qwen3 2 tokens gate_up
-// 22 / 17, 6 tokens 30 / 25 and down 18.7 / 16.6).  Four or five units a CU
+// 22 / 17, 6 tokens 30 / 25 and down 18.7 / 16.6).  At three a CU 12 waves in
+// one round are its equal or a percent faster where that round is filled
+// (Qwen3 7, 8, 9, 10 tokens gate_up 30.2 / 29.5, 31.1 / 31.2, 33.1 / 33.8, 35.1
+// / 35.7) and slower where it is not or runs over (6 tokens 29.7 / 25.4; 1536 x
+// 1024, 12 tokens 25.7 / 24.1, 14 28.4 / 21.3; 2048 x 1408, 5 tokens 30.3 / 30.2,
+// 7 45.6 / 30.5).  Four or five units a CU
 // start a second round for a part of the CUs (Qwen3 12 tokens gate_up 39 /
 // 48, 8 tokens down 19.2 / 22.4), and with short rows more rounds lose (K =
 // 768: 34.8 / 36.3 us at batch 32).  Ties keep the earlier shape in the list.
@@ -1104,13 +1109,10 @@ static PrefillShape prefill_shape(int fdim, int kdim, int planes, int tiles_hint
         const int64_t units = (int64_t)tiles_hint * pdiv_up(fdim, 32 * sh.waves);
         const int64_t per_cu = (units + c - 1) / c;
         const bool shared = sh.waves == 8 && sh.depth == 2 && 2 * lds <= kPrefillLdsMax && per_cu >= 2;
-        // Three a CU with rows of at most 2048: no better than 12 waves in one
-        // round (Qwen3 8 tokens, gate_up 31.0 / 31.4 us; in a stack 2% slower).
-        const int four = per_cu == 3 && kdim <= 2048 ? 82 : 66;
         if (sh.waves == 4 && (3 * lds > kPrefillLdsMax || (per_cu > 3 && (per_cu < 6 || kdim < 2048))))
             continue;
         // In tenths: 8, 7 for the shared 8x2 form, 6.6 for the 4-wave form.
-        const int64_t cost = per_cu * 32 * sh.waves * (sh.waves == 4 ? four : shared ? 70 : 80);
+        const int64_t cost = per_cu * 32 * sh.waves * (sh.waves == 4 ? 66 : shared ? 70 : 80);
         if (best_cost < 0 || cost < best_cost) {
             best = sh;
             best_cost = cost;
