@@ -3,6 +3,8 @@ kernels order their loads with counted vmcnt waits (a register spill adds
 scratch loads and stores to that count) and fails when one of them spills a
 vector register.  These checks run the report parser and the remark filter on
 text in the compiler's format.  CPU only."""
+import os
+
 from godwit_amd import build as gwbuild
 
 REPORT = """\
@@ -52,6 +54,16 @@ def test_without_remarks_keeps_other_diagnostics():
 def test_no_spill_sources_are_the_counted_wait_kernels():
     assert gwbuild.NO_SPILL == {"gw_decode.hip", "gw_prefill.hip"}
     assert gwbuild.NO_SPILL <= set(gwbuild.SOURCES)
+
+
+def test_spill_checked_sources_are_every_counted_wait_kernel():
+    """The build checks the sources that limit vmcnt themselves, and no kernel source that
+    does so is left out."""
+    assert gwbuild.SPILL_CHECKED == {"gw_decode.hip", "gw_prefill.hip", "gw_prefill_wide.hip"}
+    for name in gwbuild.SOURCES:
+        with open(os.path.join(gwbuild.CSRC, name)) as f:
+            counts = "wait_vmcnt<" in f.read()
+        assert not counts or name in gwbuild.SPILL_CHECKED, name
 
 
 def test_spill_check_fails_without_kernel_records():
