@@ -986,8 +986,6 @@ extern "C" int gw_expert_apply_assignments(gw_expert_runner *r, const void *inpu
     return GW_OK;
 }
 
-static size_t align256(size_t v) { return (v + 255) & ~(size_t)255; }
-
 // ---------------------------------------------------------------------------
 // MoE layer (device-routed)
 // ---------------------------------------------------------------------------
@@ -1177,6 +1175,8 @@ struct PrefillScratch {
     float *y;
     uint32_t *arrive;   // prefill_arrive_count(T, hidden) combine counters, zero between launches
 };
+
+size_t align256(size_t v) { return (v + 255) & ~(size_t)255; }
 
 // Carves the runner's prefill buffer; returns the bytes needed for (T, K, E).
 size_t prefill_layout(const gw_expert_runner *r, int T, int K, int E, char *base,

@@ -221,8 +221,6 @@ hipError_t launch_prefill_split(const Launch &L, const float *in, int64_t n, uin
 // tiles_hint: about the work list's length, used to size the workgroups.
 hipError_t launch_prefill_gemm(const Launch &L, bool gate_up, int planes, const PrefillGemm &g,
                                int max_tiles, int tiles_hint);
-// Whether launch_prefill_gemm takes inputs kdim wide (the LDS staging holds them).
-bool prefill_gemm_fits(int planes, int kdim);
 hipError_t launch_prefill_combine(const Launch &L, const float *y, const float *w, int T, int K,
                                   int H, float *out, uint16_t *out_bf16, int residual);
 

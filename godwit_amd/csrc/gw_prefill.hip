@@ -1298,11 +1298,6 @@ hipError_t launch_prefill_gemm(const Launch &L, bool gate_up, int planes, const 
     return hipGetLastError();
 }
 
-bool prefill_gemm_fits(int planes, int kdim)
-{
-    return prefill_gemm_lds_bytes(planes, kdim, 8, planes == 3 ? 2 : 4) <= kPrefillLdsMax;
-}
-
 hipError_t launch_prefill_combine(const Launch &L, const float *y, const float *w, int T, int K,
                                   int H, float *out, uint16_t *out_bf16, int residual)
 {
