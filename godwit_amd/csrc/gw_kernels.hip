@@ -810,9 +810,10 @@ __global__ __launch_bounds__(256) void router_rows_kernel(const void *__restrict
 // matrix cores: Qwen3 (128 experts) 128 tokens 17 / 10, 1021 107 / 12, 4096 421
 // / 27; GPT-OSS 128 experts 64 tokens 12 / 20, 128 17 / 18, 512 61 / 17; 32
 // experts 128 tokens 7 / 18, 512 18 / 17, 1021 33 / 18: from 16384 logits.
-// What bounds it is the texture path: a load gives 32 bytes of each of 32 rows.
-// Every load of a wave in flight, past-the-end ones clamped, was slower (15 us
-// at 1021 Qwen3 tokens).
+// What is left is latency, a launch and two dependent rounds of loads (at 1021
+// Qwen3 tokens the texture path is busy a fifth of the cycles, the matrix cores
+// 2%); with every load of a wave in flight, past-the-end ones clamped, it was
+// slower (15 us there).
 template <int XDT>
 __global__ __launch_bounds__(1024) void router_mfma_kernel(const uint16_t *__restrict__ W,
                                                            const void *__restrict__ b, int b_dt,

@@ -513,9 +513,10 @@ __global__ __launch_bounds__(64 * W, W == 8 && D == 2 ? 4 : W == 4 ? 3 : 1) void
     // run in groups of G whose B reads are issued one group ahead, and
     // alternate between two accumulators so consecutive MFMAs are independent.
     // For an fp16 x (13-bit products, CHUNKED) they sum the chunk from zero
-    // (acc1) and the chunk's sum is added to acc: with two running sums the
-    // error of a layer against 64 bits was 1.07e-5 (61 GPT-OSS tokens; 6.7e-6
-    // with the VALU dots, 8.7e-6 so), for about 1% of the time.
+    // (acc1) and the chunk's sum is added to acc: sums of 2880 products are then
+    // 8.7e-8 of their RMS from 64 bits (2048: 7.8e-8), where two running sums
+    // gave 1.50e-7 and x as two bf16 planes, the high one in one running sum,
+    // 1.11e-7 (9.2e-8); for about 1% of the time.
     constexpr int G = PL == 1 ? 4 : 1;
     constexpr int NG = 16 / G;
     // FB: the wave's scale bytes leave the fp16 range (F16IN only).  wsrc:
