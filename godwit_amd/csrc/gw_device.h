@@ -384,7 +384,9 @@ __device__ __forceinline__ void load8_f32(const void *p, int64_t i, float (&v)[8
 // 256 threads, thread t the elements t, t + 256, ... (at most NV of them, all
 // loads in flight at once): its squares in order, an xor butterfly over the
 // wave, the four wave sums in pairs.  The norm kernel and the one-token layer
-// share these steps, so both give the same bits.
+// share these steps, so both give the same bits; the squares are added by
+// explicit fused steps, since for a sum of two products written as such the
+// compiler may round either first.
 
 template <int NV>
 __device__ __forceinline__ void norm_load(const float *row, const void *weight, int w_dt, int width,
@@ -408,7 +410,7 @@ template <int NV> __device__ __forceinline__ float norm_wave_sum(const float (&v
 #pragma unroll
     for (int j = 0; j < NV; ++j) {
         const float x = t + 256 * j < width ? v[j] : 0.0f;
-        ss += x * x;
+        ss = __builtin_fmaf(x, x, ss);
     }
 #pragma unroll
     for (int o = 32; o > 0; o >>= 1) ss += __shfl_xor(ss, o);

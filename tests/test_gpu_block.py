@@ -15,7 +15,7 @@ import pytest
 
 import godwit_amd as gw
 import oracle
-from helpers import expert_metric, rng
+from helpers import expert_metric, fill_layer_device, rng
 from test_gpu_expert import GPTOSS, QWEN3, SMALL, _make_layer
 
 pytestmark = pytest.mark.gpu
@@ -152,3 +152,59 @@ def test_block_graph_replay(ctx):
     for b in (sb, wb, lb, buf):
         b.free()
     runner.close()
+
+
+def _norm_steps(stream, weight, eps):
+    """The device's RMSNorm in its own steps: thread t of 256 adds the squares of elements t,
+    t + 256, ... by fused multiply-adds from zero, an xor butterfly adds a wave's 64 sums, the
+    four waves' sums meet in pairs.  (fp32 products are exact in float64.)"""
+    T, H = stream.shape
+    x = np.zeros((T, -(-H // 256) * 256), np.float32)
+    x[:, :H] = stream
+    ss = np.zeros((T, 256), np.float32)
+    for j in range(0, x.shape[1], 256):
+        v = x[:, j:j + 256].astype(np.float64)
+        ss = (v * v + ss.astype(np.float64)).astype(np.float32)
+    for o in (32, 16, 8, 4, 2, 1):
+        ss = ss + ss[:, np.arange(256) ^ o]
+    total = (ss[:, 0] + ss[:, 64]) + (ss[:, 128] + ss[:, 192])
+    inverse = np.float32(1.0) / np.sqrt(total / np.float32(H) + np.float32(eps))
+    scaled = (stream * inverse[:, None]).astype(np.float64) * weight.astype(np.float64)
+    return scaled.astype(np.float16)
+
+
+@pytest.mark.parametrize("H,F,act,E,K,T", [
+    (2880, 2880, "gptOssClampedGLU", 8, 4, 1), (2048, 768, "silu", 16, 4, 1),   # in the layer
+    (2880, 128, "gptOssClampedGLU", 4, 2, 512), (2080, 128, "silu", 4, 2, 512),  # the norm kernel
+], ids=["2880-t1", "2048-t1", "2880-t512", "2080-t512"])
+def test_norm_bits(ctx, H, F, act, E, K, T):
+    """The block's normalised rows are the bits that the norm's steps give, wherever it runs:
+    a block's stream is the stream plus the layer's output on the rows made so on the host."""
+    eps, rows = 1e-5, 512
+    r = rng(9200 + H + T)
+    layout = gw.ExpertLayout(H, F, E)
+    buf = ctx.empty(layout.layer_file_size)
+    fill_layer_device(ctx, buf, layout, E, 9201)
+    for sec in ("gate_up_scales", "down_scales"):
+        ctx.fill_uniform_u8(buf, 117, 122, 9202, offset=layout.offsets[sec],
+                            count=layout.sizes[sec], rows=E, row_stride=layout.stride)
+    wbits = _norm_weight(r, H)
+    stream = (4.0 * r.standard_normal((rows, H))).astype(np.float32)
+    x = _norm_steps(stream, oracle.bf16_bits_to_f32(wbits), eps)
+    logits = r.standard_normal((rows, E)).astype(np.float32)
+    sb, xb, wb, lb = ctx.buffer(stream), ctx.buffer(x), ctx.buffer(wbits), ctx.buffer(logits)
+    out = ctx.empty(rows * H * 4)
+    runner = gw.ExpertRunner(ctx, H, F, act)
+    for t in range(0, rows, T):
+        runner.layer_forward(buf.ptr, layout.stride, E, K, xb.ptr + t * H * 2, gw.F16, T,
+                             out.ptr + t * H * 4, logits=lb.ptr + t * E * 4)
+        runner.block_forward(buf.ptr, layout.stride, E, K, T, sb.ptr + t * H * 4, wb.ptr, eps,
+                             logits=lb.ptr + t * E * 4)
+    ctx.synchronize()
+    moe = out.download(np.float32, rows * H).reshape(rows, H)
+    got = sb.download(np.float32, rows * H).reshape(rows, H)
+    bad = np.nonzero((got != stream + moe).any(1))[0]
+    assert len(bad) == 0, bad
+    runner.close()
+    for b in (sb, xb, wb, lb, out, buf):
+        b.free()
