@@ -802,11 +802,14 @@ __global__ __launch_bounds__(256) void router_rows_kernel(const void *__restrict
 
 // Router logits of a batch with bf16 weights and 16-bit x on the matrix cores:
 // workgroup (32 tokens, 32 experts), its 16 waves a sixteenth of K each, whose
-// partial tiles meet in LDS and are added in wave order plus the bias.  The
-// products are exact (an fp16 x enters as hi + lo, two bf16 values whose sum it
-// is; infinities and NaN give what one product would), a wave's sum is a few
-// MFMA steps long.  router_rows_kernel reads a
-// weight row for each 8 tokens with one product a lane-op.  us a launch, rows /
+// partial tiles meet in LDS and are added, with the bias, in fp64.  The products
+// are exact (an fp16 x enters as hi + lo, two bf16 values whose sum it is;
+// infinities and NaN give what one product would); a wave adds them up in two
+// sums a few MFMA steps long, and lo's in a third.  2880 fp16 products are then
+// 6.7e-8 of their RMS from 64 bits, bf16 6.2e-8 (router_rows_kernel 8.5e-8 and
+// 7.5e-8; one sum a wave and fp32 between them 1.34e-7 and 1.05e-7).
+// router_rows_kernel reads a weight row for each 8 tokens with one product a
+// lane-op.  us a launch, rows /
 // matrix cores: Qwen3 (128 experts) 128 tokens 17 / 10, 1021 107 / 12, 4096 421
 // / 27; GPT-OSS 128 experts 64 tokens 12 / 20, 128 17 / 18, 512 61 / 17; 32
 // experts 128 tokens 7 / 18, 512 18 / 17, 1021 33 / 18: from 16384 logits.
@@ -832,13 +835,17 @@ __global__ __launch_bounds__(1024) void router_mfma_kernel(const uint16_t *__res
     const uint16_t *xr = x + (int64_t)min(t0 + c, T - 1) * H + 8 * h;
     const int steps = H >> 4;
     const int s0 = wave * steps / kWaves, s1 = (wave + 1) * steps / kWaves;
-    f32x16 acc;
+    // Steps in turn into two sums, the lo products of an fp16 x into a third.
+    constexpr int kSums = XDT == DT_BF16 ? 2 : 3;
+    f32x16 acc[kSums];
     // NONFINITE: an infinite x is its hi alone (v - hi would be NaN), and an
     // infinite or NaN weight meets no lo (which is 0 where x is its hi).
     auto add_up = [&](auto nonfinite) {
         constexpr bool NONFINITE = decltype(nonfinite)::value;
 #pragma unroll
-        for (int v = 0; v < 16; ++v) acc[v] = 0.0f;
+        for (int k = 0; k < kSums; ++k)
+#pragma unroll
+            for (int v = 0; v < 16; ++v) acc[k][v] = 0.0f;
         for (int s = s0; s < s1; s += kU) {
             uint4 a[kU], v[kU];
 #pragma unroll
@@ -852,7 +859,8 @@ __global__ __launch_bounds__(1024) void router_mfma_kernel(const uint16_t *__res
                 if (s + u >= s1) break;               // uniform
                 const bf16x8 aw = __builtin_bit_cast(bf16x8, a[u]);
                 if constexpr (XDT == DT_BF16) {
-                    acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(aw, __builtin_bit_cast(bf16x8, v[u]), acc, 0, 0, 0);
+                    acc[u & 1] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
+                        aw, __builtin_bit_cast(bf16x8, v[u]), acc[u & 1], 0, 0, 0);
                 } else {
                     const uint32_t r[4] = {v[u].x, v[u].y, v[u].z, v[u].w};
                     uint32_t wl[4] = {a[u].x, a[u].y, a[u].z, a[u].w};
@@ -873,14 +881,18 @@ __global__ __launch_bounds__(1024) void router_mfma_kernel(const uint16_t *__res
                             if ((wl[k] & 0x7F800000u) == 0x7F800000u) wl[k] &= 0x0000FFFFu;
                         }
                     }
-                    acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
+                    acc[2] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
                         __builtin_bit_cast(bf16x8, make_uint4(wl[0], wl[1], wl[2], wl[3])),
-                        __builtin_bit_cast(bf16x8, make_uint4(lo[0], lo[1], lo[2], lo[3])), acc, 0, 0, 0);
-                    acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
-                        aw, __builtin_bit_cast(bf16x8, make_uint4(hi[0], hi[1], hi[2], hi[3])), acc, 0, 0, 0);
+                        __builtin_bit_cast(bf16x8, make_uint4(lo[0], lo[1], lo[2], lo[3])), acc[2], 0, 0, 0);
+                    acc[u & 1] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
+                        aw, __builtin_bit_cast(bf16x8, make_uint4(hi[0], hi[1], hi[2], hi[3])), acc[u & 1], 0, 0, 0);
                 }
             }
         }
+    };
+    auto total = [&](int v) {
+        const float hi = acc[0][v] + acc[1][v];
+        return XDT == DT_BF16 ? hi : hi + acc[kSums - 1][v];
     };
     add_up(std::false_type{});
     if constexpr (XDT == DT_F16) {
@@ -888,21 +900,21 @@ __global__ __launch_bounds__(1024) void router_mfma_kernel(const uint16_t *__res
         // is the share summed once more (a check of every step took 4 us).
         bool finite = true;
 #pragma unroll
-        for (int v = 0; v < 16; ++v) finite &= fabsf(acc[v]) < __builtin_inff();
+        for (int v = 0; v < 16; ++v) finite &= fabsf(total(v)) < __builtin_inff();
         if (__ballot(!finite)) add_up(std::true_type{});
     }
 #pragma unroll
     for (int v = 0; v < 16; ++v) {
         const int e = 8 * (v >> 2) + 4 * h + (v & 3);
-        part[wave][32 * e + (c ^ e)] = acc[v];
+        part[wave][32 * e + (c ^ e)] = total(v);
     }
     __syncthreads();
     const int e = (int)threadIdx.x & 31, t = (int)threadIdx.x >> 5;
-    float sum = part[0][32 * e + (t ^ e)];
+    double sum = 0.0;
 #pragma unroll
-    for (int w = 1; w < kWaves; ++w) sum += part[w][32 * e + (t ^ e)];
+    for (int w = 0; w < kWaves; ++w) sum += (double)part[w][32 * e + (t ^ e)];
     if (e0 + e < E && t0 + t < T)
-        logits[(int64_t)(t0 + t) * E + e0 + e] = sum + load_bias(b, b_dt, e0 + e);
+        logits[(int64_t)(t0 + t) * E + e0 + e] = (float)(sum + (double)load_bias(b, b_dt, e0 + e));
 }
 
 // Router logits of one token by slices (router_partial, the same order as the

@@ -417,3 +417,33 @@ def test_router_logits_batch_non_finite(ctx, x_dtype):
         assert np.all(np.abs(got[finite] - want[finite]) <= size[finite] * 2.0 ** -20)
     for b in (wbuf, xbuf, out):
         b.free()
+
+
+@pytest.mark.parametrize("experts,hidden,tokens", [(128, 2048, 256), (32, 2880, 512)])
+@pytest.mark.parametrize("x_dtype", [gw.F16, gw.BF16], ids=["f16", "bf16"])
+def test_router_logits_batch_error(ctx, experts, hidden, tokens, x_dtype):
+    """A batch's logits on the matrix cores are no further from float64, in RMS over its
+    16384 logits, than the same rows taken 8 at a time."""
+    r = rng(7900 + hidden)
+    wb = oracle.f32_to_bf16_bits((0.02 * r.standard_normal(experts * hidden)).astype(np.float32))
+    w = oracle.bf16_bits_to_f32(wb).astype(np.float64).reshape(experts, hidden)
+    x = r.standard_normal((tokens, hidden)).astype(np.float32)
+    if x_dtype == gw.F16:
+        xb = x.astype(np.float16)
+        x = xb.astype(np.float64)
+    else:
+        xb = oracle.f32_to_bf16_bits(x.ravel())
+        x = oracle.bf16_bits_to_f32(xb).astype(np.float64).reshape(tokens, hidden)
+    wbuf, xbuf, out = ctx.buffer(wb), ctx.buffer(xb), ctx.empty(tokens * experts * 4)
+
+    def logits(t0, n):
+        check(lib.gw_router_logits(ctx.handle, wbuf.ptr, gw.BF16, None, gw.BF16,
+                                   xbuf.ptr + t0 * hidden * 2, x_dtype, out.ptr, experts, hidden, n))
+        return out.download(np.float32, n * experts).reshape(n, experts)
+
+    want = x @ w.T
+    rms = [np.sqrt(np.mean((got - want) ** 2)) for got in (
+        logits(0, tokens), np.concatenate([logits(t, 8) for t in range(0, tokens, 8)]))]
+    assert rms[0] <= rms[1], rms
+    for b in (wbuf, xbuf, out):
+        b.free()
