@@ -1052,17 +1052,21 @@ static int moe_layer_impl(gw_expert_runner *r, const gw_moe_layer_args *a, int o
     // router rows split evenly over its grid (16-bit x, up to 128 experts).
     gw::DecodeArgs d = {};
     size_t dlds = 0;
-    const int dgrid = a->tokens == 1 && r->decode_layer
-                          ? gw::decode_layer_plan(L, (int)r->hidden, (int)r->inter, a->x_dtype,
-                                                  (int)a->top_k, (int)a->expert_count,
-                                                  a->expert_stride, r->bias_dt, &d, &dlds)
-                          : 0;
+    auto plan = [&](bool with_norm) {
+        return a->tokens == 1 && r->decode_layer
+                   ? gw::decode_layer_plan(L, (int)r->hidden, (int)r->inter, a->x_dtype,
+                                           (int)a->top_k, (int)a->expert_count,
+                                           a->expert_stride, r->bias_dt, with_norm, &d, &dlds)
+                   : 0;
+    };
+    int dgrid = plan(norm != nullptr);
     const int rslices = dgrid > 0 && !a->logits && a->expert_count <= 128 &&
                                 aligned16(a->router_weight) && aligned16(a->x)
                             ? gw::router_slices((int)a->expert_count, (int)r->hidden, dgrid)
                             : 0;
     const bool fused_norm = norm && dgrid > 0 && (a->logits || rslices > 0);
-    if (!fused_norm) {
+    if (!fused_norm && norm) {
+        dgrid = plan(false);
         int rc = run_norm();
         if (rc) return rc;
     }

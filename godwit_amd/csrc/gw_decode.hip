@@ -220,8 +220,8 @@ __device__ __forceinline__ uint32_t pair_empty(const u32x4 &v)
 // blocks each.  NSP: 1 KiB pieces of down scale bytes each DMA wave copies.  PD: ticks of the 100 MHz real-time counter between the
 // workgroup publishing its activations and its first read of the exchange.
 // PX: a gate_up wave reads its DMA partner's exchange words into LDS (else
-// every wave reads its own).
-template <int XK, class GS, int NSG, int GD, int TD, int WT, int SPW, int NSP, int PD, bool PX>
+// every wave reads its own).  NORM: the row is a.stream's, normalised here.
+template <int XK, class GS, int NSG, int GD, int TD, int WT, int SPW, int NSP, int PD, bool PX, bool NORM>
 __global__ __launch_bounds__(kDT) void decode_layer_kernel(DecodeArgs a)
 {
     constexpr int TPG = GS::TPR, MG = GS::M, SEGG = 64 / TPG, RGW = kGuWaves * SEGG;
@@ -291,37 +291,35 @@ __global__ __launch_bounds__(kDT) void decode_layer_kernel(DecodeArgs a)
     // costs: with a norm kernel in front a block took 29.8 us a layer (GPT-OSS,
     // 32 experts, replayed; 9.4 of them that kernel) and 21.1 (Qwen3), with
     // the row in registers here 21.7 and 14.6.
-    if constexpr (XK == DT_F16) {
-        if (a.norm_w) {                               // uniform
-            constexpr int NV = GS::M == 6 ? 12 : 8;   // 96 or 64 blocks of 32 over 256 threads
-            float *sums = reinterpret_cast<float *>(lds8 + L.route + 192);
-            const int t = (int)threadIdx.x;
-            float v[NV], w[NV];
-            if (wave < 4) {
-                norm_load<NV>(a.stream, a.norm_w, a.norm_dt, H, t, v, w);
-                const float ss = norm_wave_sum<NV>(v, H, t);
-                if (lane == 0) sums[wave] = ss;
-            } else if (wave == 4 && a.rw) {
-                const int Lw = H / a.rslices, esz = a.rw_dt == DT_F32 ? 4 : 2;
-                const char *p = static_cast<const char *>(a.rw) +
-                                ((int64_t)(b / a.rslices) * H + (int64_t)(b % a.rslices) * Lw) * esz;
-                for (int i = lane * 64; i < Lw * esz; i += 64 * 64) {
-                    const uint32_t touch = *reinterpret_cast<const uint32_t *>(p + i);
-                    asm volatile("" : : "v"(touch));
-                }
+    if constexpr (NORM) {
+        constexpr int NV = GS::M == 6 ? 12 : 8;   // 96 or 64 blocks of 32 over 256 threads
+        float *sums = reinterpret_cast<float *>(lds8 + L.route + 192);
+        const int t = (int)threadIdx.x;
+        float v[NV], w[NV];
+        if (wave < 4) {
+            norm_load<NV>(a.stream, a.norm_w, a.norm_dt, H, t, v, w);
+            const float ss = norm_wave_sum<NV>(v, H, t);
+            if (lane == 0) sums[wave] = ss;
+        } else if (wave == 4 && a.rw) {
+            const int Lw = H / a.rslices, esz = a.rw_dt == DT_F32 ? 4 : 2;
+            const char *p = static_cast<const char *>(a.rw) +
+                            ((int64_t)(b / a.rslices) * H + (int64_t)(b % a.rslices) * Lw) * esz;
+            for (int i = lane * 64; i < Lw * esz; i += 64 * 64) {
+                const uint32_t touch = *reinterpret_cast<const uint32_t *>(p + i);
+                asm volatile("" : : "v"(touch));
             }
-            __syncthreads();
-            if (wave < 4) {
-                const float inverse = norm_inverse(sums, H, a.norm_eps);
-                uint16_t *x16 = reinterpret_cast<uint16_t *>(xs);
-#pragma unroll
-                for (int j = 0; j < NV; ++j) {
-                    const int i = t + 256 * j;
-                    if (i < H) x16[(i >> 5) * (BD * 2) + (i & 31)] = f32_to_f16_bits((v[j] * inverse) * w[j]);
-                }
-            }
-            __syncthreads();
         }
+        __syncthreads();
+        if (wave < 4) {
+            const float inverse = norm_inverse(sums, H, a.norm_eps);
+            uint16_t *x16 = reinterpret_cast<uint16_t *>(xs);
+#pragma unroll
+            for (int j = 0; j < NV; ++j) {
+                const int i = t + 256 * j;
+                if (i < H) x16[(i >> 5) * (BD * 2) + (i & 31)] = f32_to_f16_bits((v[j] * inverse) * w[j]);
+            }
+        }
+        __syncthreads();
     }
     if (wave == 0) {
         if (by_rank) {
@@ -335,7 +333,7 @@ __global__ __launch_bounds__(kDT) void decode_layer_kernel(DecodeArgs a)
                 // logit its partials in slice order plus the bias.
                 const int S = a.rslices, Lw = H / S;
                 float p;
-                if (XK == DT_F16 && a.norm_w)
+                if constexpr (NORM)
                     p = router_partial_lds_dt(a.rw, a.rw_dt, xs, b / S, b % S, Lw, H, lane);
                 else
                     p = router_partial_dt<XK>(a.rw, a.rw_dt, a.x, b / S, b % S, Lw, H, lane);
@@ -424,7 +422,7 @@ __global__ __launch_bounds__(kDT) void decode_layer_kernel(DecodeArgs a)
                 if (b == 0 && a.w_out) a.w_out[lane] = w;
             }
         }
-    } else if (XK != DT_F16 || !a.norm_w) {
+    } else if (!NORM) {
         stage_vector<XK>(xs, a.x, H, threadIdx.x - 64, kDT - 64);
     }
     __syncthreads();
@@ -1110,31 +1108,34 @@ int shape_of(int hidden, int inter)
     return -1;
 }
 
-#define GW_DECODE_KERNEL(S, XD)                                                                 \
+#define GW_DECODE_KERNEL(S, XD, N)                                                              \
     decode_layer_kernel<XD, DShape<16, (S) == kShapeGptOss ? 6 : 4>, kStagesG[S], kRingG[S], kTiles[S], \
-                        kTileGroups[S], kStepsPerWave[S], kScalePieces[S], kPollDelay[S], kPartnerReads[S]>
+                        kTileGroups[S], kStepsPerWave[S], kScalePieces[S], kPollDelay[S], kPartnerReads[S], N>
 
 typedef void (*DecodeKernel)(DecodeArgs);
 
-// The instantiation for (shape, x dtype).
-DecodeKernel kernel_for(int shape, int x_dt)
+// The instantiation for (shape, x dtype, norm in the kernel).  The norm has
+// instantiations of its own: as a branch it cost a layer without it 1.5%.
+DecodeKernel kernel_for(int shape, int x_dt, bool norm)
 {
     if (shape == kShapeGptOss)
-        return x_dt == DT_BF16 ? &GW_DECODE_KERNEL(kShapeGptOss, DT_BF16)
-                               : &GW_DECODE_KERNEL(kShapeGptOss, DT_F16);
-    return x_dt == DT_BF16 ? &GW_DECODE_KERNEL(kShapeQwen3, DT_BF16)
-                           : &GW_DECODE_KERNEL(kShapeQwen3, DT_F16);
+        return x_dt == DT_BF16 ? &GW_DECODE_KERNEL(kShapeGptOss, DT_BF16, false)
+               : norm          ? &GW_DECODE_KERNEL(kShapeGptOss, DT_F16, true)
+                               : &GW_DECODE_KERNEL(kShapeGptOss, DT_F16, false);
+    return x_dt == DT_BF16 ? &GW_DECODE_KERNEL(kShapeQwen3, DT_BF16, false)
+           : norm          ? &GW_DECODE_KERNEL(kShapeQwen3, DT_F16, true)
+                           : &GW_DECODE_KERNEL(kShapeQwen3, DT_F16, false);
 }
 
 }  // namespace
 #undef GW_DECODE_KERNEL
 
 int decode_layer_plan(const Launch &L, int hidden, int inter, int x_dt, int top_k, int experts,
-                      int64_t stride, int bias_dt, DecodeArgs *args, size_t *lds_bytes)
+                      int64_t stride, int bias_dt, bool norm, DecodeArgs *args, size_t *lds_bytes)
 {
     (void)bias_dt;
     const int shape = shape_of(hidden, inter);
-    if (shape < 0 || (x_dt != DT_BF16 && x_dt != DT_F16)) return 0;
+    if (shape < 0 || (x_dt != DT_BF16 && x_dt != DT_F16) || (norm && x_dt != DT_F16)) return 0;
     if (top_k < 1 || top_k > kMaxTopK || experts > 256 || experts < top_k) return 0;
     if ((int64_t)experts * stride >= (int64_t)kOutOfRange) return 0;   // 32-bit buffer offsets
     const int G = L.cus;
@@ -1157,10 +1158,10 @@ int decode_layer_plan(const Launch &L, int hidden, int inter, int x_dt, int top_
                                    kPartnerReads[shape] ? (8 - kGuWaves) * spw * 4 : 0);
     if (l.total > kDecodeLdsMax) return 0;
     // The exchange needs the whole grid resident: one workgroup per CU.
-    const void *fn = reinterpret_cast<const void *>(kernel_for(shape, x_dt));
-    static const void *attr_done[4] = {};
+    const void *fn = reinterpret_cast<const void *>(kernel_for(shape, x_dt, norm));
+    static const void *attr_done[6] = {};
     int slot = -1;
-    for (int i = 0; i < 4; ++i)
+    for (int i = 0; i < 6; ++i)
         if (attr_done[i] == fn || attr_done[i] == nullptr) { slot = i; break; }
     if (slot < 0) return 0;
     if (attr_done[slot] != fn) {
@@ -1185,7 +1186,7 @@ hipError_t launch_decode_layer(const Launch &L, int grid, size_t lds, int x_dt, 
 {
     const int shape = shape_of(a.hidden, a.inter);
     if (shape < 0 || grid <= 0) return hipErrorInvalidValue;
-    const DecodeKernel kernel = kernel_for(shape, x_dt);
+    const DecodeKernel kernel = kernel_for(shape, x_dt, a.norm_w != nullptr);
     if (L.coop && !L.ev_start) {
         DecodeArgs copy = a;
         void *args[] = {&copy};

@@ -133,9 +133,10 @@ struct DecodeLds { int route, xs, actl, dma, scl, part, bx, total; };
 
 // Grid (one workgroup per CU) of the one-kernel layer for this shape, or 0
 // when it is not available (shape, dtype or top-k not built, LDS, or the grid
-// cannot be resident).  Fills args->nrmax / base_bytes and the LDS size.
+// cannot be resident).  norm: the kernel with the RMSNorm in it.  Fills
+// args->nrmax / base_bytes and the LDS size.
 int decode_layer_plan(const Launch &L, int hidden, int inter, int x_dt, int top_k, int experts,
-                      int64_t stride, int bias_dt, DecodeArgs *args, size_t *lds_bytes);
+                      int64_t stride, int bias_dt, bool norm, DecodeArgs *args, size_t *lds_bytes);
 hipError_t launch_decode_layer(const Launch &L, int grid, size_t lds, int x_dt,
                                const DecodeArgs &a);
 // ---- prefill (batched tokens) on the matrix cores
