@@ -1350,7 +1350,8 @@ static int moe_prefill_impl(gw_expert_runner *r, const gw_moe_layer_args *a, int
         !wide &&
         (T <= r->fused_combine_max ||
          (r->fused_combine_max > 0 &&
-          gw::prefill_down_four_wave((int)r->hidden, (int)r->inter, hint, max_tiles, L.cus))) &&
+          gw::prefill_down_four_wave((int)r->hidden, (int)r->inter, hint, max_tiles, L.cus,
+                                     self_group))) &&
         (int64_t)sizeof(float) * T * K * r->hidden < ((int64_t)1 << 31);
     gw::PrefillGemm g;
     g.wide = wide;

@@ -810,7 +810,7 @@ __global__ __launch_bounds__(256) void router_rows_kernel(const void *__restrict
 // 7.5e-8; one sum a wave and fp32 between them 1.34e-7 and 1.05e-7).
 // router_rows_kernel reads a weight row for each 8 tokens with one product a
 // lane-op.  us a launch, rows /
-// matrix cores: Qwen3 (128 experts) 128 tokens 17 / 10, 1021 107 / 12, 4096 421
+// matrix cores: Qwen3 (128 experts) 128 tokens 17 / 10, 1021 112 / 14, 4096 421
 // / 27; GPT-OSS 128 experts 64 tokens 12 / 20, 128 17 / 18, 512 61 / 17; 32
 // experts 128 tokens 7 / 18, 512 18 / 17, 1021 33 / 18: from 16384 logits.
 // What is left is latency, a launch and two dependent rounds of loads (at 1021

@@ -1072,28 +1072,30 @@ int prefill_gemm_lds_bytes(int planes, int kdim, int waves, int depth)
 // 426 -> 403 us), while one workgroup per CU runs better with a 4-deep ring
 // (a 12-wave gate_up that fits the CUs in one round: 35 against 40 us).  The
 // 4-wave, 2-deep form (one plane: 45 KB of LDS at K = 2880, three workgroups
-// per CU) is priced at 6.6 where each CU takes at least six of its units and
-// K spans at least eight chunks (three independent workgroups overlap one
-// another's weight waits better still: 512 tokens, gate_up 382 -> 365 us,
-// down 208 -> 192 us; Qwen3 batch 32 gate_up 51.9 -> 49.8 us), and where all
-// of its units are resident at once, at most three a CU: the work is then
-// spread by 128 rows instead of 256 (us, the other shapes / this; GPT-OSS 2
-// tokens down 26 / 20, 6 tokens down 46 / 35, 4 tokens gate_up 42 / 40, fp16
-// 47 / 40, 16 fp16 tokens of 32 experts down 47 / 38; Qwen3 2 tokens gate_up
-// 22 / 17, 6 tokens 30 / 25 and down 18.7 / 16.6).  At three a CU 12 waves in
-// one round are its equal or a percent faster where that round is filled
-// (Qwen3 7, 8, 9, 10 tokens gate_up 30.2 / 29.5, 31.1 / 31.2, 33.1 / 33.8, 35.1
-// / 35.7) and slower where it is not or runs over (6 tokens 29.7 / 25.4; 1536 x
-// 1024, 12 tokens 25.7 / 24.1, 14 28.4 / 21.3; 2048 x 1408, 5 tokens 30.3 / 30.2,
-// 7 45.6 / 30.5).  Four or five units a CU
-// start a second round for a part of the CUs (Qwen3 12 tokens gate_up 39 /
-// 48, 8 tokens down 19.2 / 22.4), and with short rows more rounds lose (K =
-// 768: 34.8 / 36.3 us at batch 32).  Ties keep the earlier shape in the list.
-// `tiles_hint` is about the length of the work list.
+// per CU) is priced at 6.6 where all of its units are resident at once, at
+// most three a CU, and where K spans at least eight chunks: the work is spread
+// by 128 rows instead of 256, and three independent workgroups overlap one
+// another's weight waits.  us, the best other shape / this, by units a CU:
+// GPT-OSS, 128 experts, 6 tokens down (2.1) 45.0 / 35.9, 14 (4.2) 68.0 / 55.8, 16
+// (4.8) 69.6 / 58.6; 32 experts, 13 tokens gate_up (4.9) 68.6 / 55.4, 32 down
+// (3.2) 47.4 / 39.0; Qwen3 gate_up, 14 tokens (3.8) 35.4 / 34.1, 20 (4.6) 48.9 /
+// 39.8, 28 (5.3) 50.1 / 43.6; 512 GPT-OSS tokens, gate_up 382 / 365, down 208 /
+// 192.  A self-grouped batch (each workgroup then finds its own work) leaves
+// it between three units a CU and 33/8, where a second round starts for a part
+// of the CUs: Qwen3 12 tokens gate_up (3.4) 39.2 / 47.7, 2048 x 1408 12 tokens
+// (4.0) 42.6 / 47.0, GPT-OSS 32 experts 8 tokens (4.0) 50.3 / 51.8, 6 (3.2) 49.5
+// / 48.6.  With shorter rows it wins and loses (K = 768, Qwen3 down, 12 tokens
+// (4.5) 27.2 / 25.0, 16 (5.4) even; K = 1408, 28 tokens down (4.1) 28.9 / 30.7).
+// At three a CU 12 waves in one round are its equal or a percent faster where
+// that round is filled (Qwen3 7, 8, 9, 10 tokens gate_up 30.2 / 29.5, 31.1 /
+// 31.2, 33.1 / 33.8, 35.1 / 35.7) and slower where it is not or runs over (6
+// tokens 29.7 / 25.4; 1536 x 1024, 14 tokens 28.4 / 21.3; 2048 x 1408, 7 tokens
+// 45.6 / 30.5).  Ties keep the earlier shape in the list.  `tiles_hint` is
+// about the length of the work list.
 struct PrefillShape { int waves, depth; };
 
 static PrefillShape prefill_shape(int fdim, int kdim, int planes, int tiles_hint, int cus,
-                                  bool twelve, bool four_waves)
+                                  bool twelve, bool four_waves, bool self_group)
 {
     const int c = cus > 0 ? cus : 1;
     const PrefillShape cand[4] = {{8, planes == 3 ? 2 : 4}, {12, planes == 3 ? 2 : 4}, {8, 2},
@@ -1110,7 +1112,8 @@ static PrefillShape prefill_shape(int fdim, int kdim, int planes, int tiles_hint
         const int64_t units = (int64_t)tiles_hint * pdiv_up(fdim, 32 * sh.waves);
         const int64_t per_cu = (units + c - 1) / c;
         const bool shared = sh.waves == 8 && sh.depth == 2 && 2 * lds <= kPrefillLdsMax && per_cu >= 2;
-        if (sh.waves == 4 && (3 * lds > kPrefillLdsMax || (per_cu > 3 && (per_cu < 6 || kdim < 2048))))
+        if (sh.waves == 4 && (3 * lds > kPrefillLdsMax ||
+                              (units > 3 * c && (kdim < 2048 || (self_group && 8 * units < 33 * c)))))
             continue;
         // In tenths: 8, 7 for the shared 8x2 form, 6.6 for the 4-wave form.
         const int64_t cost = per_cu * 32 * sh.waves * (sh.waves == 4 ? 66 : shared ? 70 : 80);
@@ -1122,10 +1125,10 @@ static PrefillShape prefill_shape(int fdim, int kdim, int planes, int tiles_hint
     return best;
 }
 
-bool prefill_down_four_wave(int fdim, int kdim, int tiles_hint, int max_tiles, int cus)
+bool prefill_down_four_wave(int fdim, int kdim, int tiles_hint, int max_tiles, int cus, bool self_group)
 {
     const int hint = tiles_hint > 0 && tiles_hint < max_tiles ? tiles_hint : max_tiles;
-    return prefill_shape(fdim, kdim, 1, hint, cus, false, true).waves == 4;
+    return prefill_shape(fdim, kdim, 1, hint, cus, false, true, self_group).waves == 4;
 }
 
 hipError_t launch_prefill_split(const Launch &L, const float *in, int64_t n, uint16_t *out)
@@ -1215,7 +1218,7 @@ hipError_t launch_prefill_gemm(const Launch &L, bool gate_up, int planes, const 
     const bool four = planes == 1;
     PrefillShape sh = prefill_shape(
         g.fdim, g.kdim, planes, tiles_hint > 0 && tiles_hint < max_tiles ? tiles_hint : max_tiles,
-        L.cus, twelve, four);
+        L.cus, twelve, four, g.sg_tokens > 0);
     if (g.force_waves == 4 && four) {
         const PrefillShape f = {4, 2};
         if (prefill_gemm_lds_bytes(planes, g.kdim, 4, 2) <= kPrefillLdsMax) sh = f;
