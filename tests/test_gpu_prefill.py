@@ -5,8 +5,8 @@ The oracle is the reference's layer: route each token (Router.select), run
 every selected expert (referenceMXFP4 GEMVs + activation with fp16 rounding)
 and combine in router order.  Tolerance: the reference's expert metric
 max|d|/mean|ref| per token (GodwitCLI/main.swift:518-532) below 1e-3, see
-_close_batch; routing ids exact, weights to 1e-6.  Shapes cover one, two and three bf16
-activation planes (bf16, fp16, fp32 x), partial feature tiles, K dimensions
+_close_batch; routing ids exact, weights to 1e-6.  Shapes cover one bf16 or fp16 plane and
+three bf16 planes (bf16, fp16, fp32 x), partial feature tiles, K dimensions
 that are not a multiple of the 256-element staging chunk, experts with no
 tokens and experts with several 32-token tiles.
 """
@@ -74,7 +74,7 @@ def _run(ctx, runner, layout, buf, E, K, xb, x_dtype, lb, T, H, fn="prefill_forw
 
 @pytest.mark.parametrize("shape,E,K,T,x_dtype,seed", [
     (SMALL, 16, 4, 72, gw.BF16, 1),      # experts with 2-3 tiles, partial feature tiles
-    (QWEN3, 32, 8, 24, gw.F16, 2),       # two activation planes, no biases, SiLU-GLU
+    (QWEN3, 32, 8, 24, gw.F16, 2),       # one fp16 plane, no biases, SiLU-GLU
     (GPTOSS, 12, 4, 20, gw.F32, 3),      # three planes, 2880-wide K (11.25 chunks)
     (SMALL, 200, 4, 32, gw.BF16, 4),     # 200 experts, 32 tokens routed in the group kernel
     (SMALL, 256, 8, 40, gw.BF16, 5),     # route kernel, then a scan over 256 experts
@@ -253,16 +253,16 @@ def test_self_grouped_equals_tile_list(ctx, monkeypatch, shape, E, K, T, x_dtype
 
 
 @pytest.mark.parametrize("shape,E,K,T,x_dtype,seed", [
-    (QWEN3, 128, 8, 8, gw.BF16, 1),      # config 3's batch: one plane in, two for down
-    (SMALL, 16, 4, 72, gw.F16, 2),       # two planes in, several tiles per expert (tile list)
+    (QWEN3, 128, 8, 8, gw.BF16, 1),      # config 3's batch: one bf16 plane in, one fp16 for down
+    (SMALL, 16, 4, 72, gw.F16, 2),       # one fp16 plane, several tiles per expert (tile list)
     (GPTOSS, 12, 4, 20, gw.F32, 3),      # three planes: 2-deep rings only
     (SMALL, 256, 8, 32, gw.BF16, 4),     # 32 KB of logits: past the 8x2 ring, read in place
 ], ids=["qwen3-t8", "small-f16-t72", "gptoss-f32-t20", "small-e256-t32"])
 def test_gemm_shapes_bit_identical(ctx, monkeypatch, shape, E, K, T, x_dtype, seed):
-    """The grouped GEMMs run 8 waves with a 4-deep ring, 12 waves (4-deep; gate_up
-    only, the down GEMM takes 8x4 instead), 8 waves with a 2-deep ring held to
+    """The grouped GEMMs run 8 waves with a 4-deep ring, 12 waves (4-deep; gate_up of a bf16
+    or fp32 x only, the other launches take 8x4 instead), 8 waves with a 2-deep ring held to
     128 VGPRs so that two workgroups share a CU, or 4 waves with a 2-deep ring
-    (gate_up with bf16 x only; three workgroups per CU); the launcher picks one
+    (bf16 and fp16 x and the down GEMM; three workgroups per CU); the launcher picks one
     per launch and GODWIT_PREFILL_SHAPE forces one at runner creation.  Every
     shape gives the same bytes (each output keeps its chunk and MFMA order),
     and the chosen one equals the oracle."""
@@ -626,8 +626,8 @@ def test_prefill_gate_up_fp16_x(ctx, monkeypatch, T, forced):
     (128, 320, gw.BF16, "silu"),               # one chunk; 10 blocks, a last chunk of 2
 ])
 def test_wide_tiles_match_oracle(ctx, monkeypatch, hidden, inter, x_dtype, act):
-    """Tiles of up to 128 entries (GODWIT_WIDE_ENTRIES=0 runs them at any size) with every
-    number of 32-entry column groups, full and with one entry, second tiles, and an expert
+    """Tiles of up to 96 entries (GODWIT_WIDE_ENTRIES=0 runs them for any batch past
+    self-grouping) with every number of 32-entry column groups, full and with one entry, second tiles, and an expert
     without entries; rows past the last feature tile and K of any number of blocks."""
     monkeypatch.setenv("GODWIT_WIDE_ENTRIES", "0")
     counts = [1, 32, 33, 64, 65, 96, 0, 97, 128, 129]
@@ -814,3 +814,44 @@ def test_wide_tiles_default_rule(ctx, shape, E, K, T):
     for b in (lb, buf):
         b.free()
     runner.close()
+
+
+@pytest.mark.parametrize("x_dtype", [gw.BF16, gw.F16], ids=["bf16", "f16"])
+@pytest.mark.parametrize("H,F,act", [(352, 224, "silu"), (1024, 512, "gptOssClampedGLU")])
+def test_wide_tiles_general_body(ctx, monkeypatch, H, F, act, x_dtype):
+    """Every row with one scale byte outside the fast range (0 for a bf16 x, 103 for an fp16 x
+    and the activations): the wide tiles take their general body, one column group after
+    another, with the split products and sums of the 32-entry tiles' own, so the bytes are
+    the same, in tiles of one to three groups and second tiles; and they agree with fp64."""
+    counts = [1, 64, 65, 96, 130, 33]
+    E, T = len(counts), sum(counts)
+    layout = gw.ExpertLayout(H, F, E)
+    r = rng(4100 + H)
+    buf = ctx.empty(layout.layer_file_size)
+    fill_layer_device(ctx, buf, layout, E, 4101)
+    raw = buf.download(np.uint8, layout.stride * E).reshape(E, layout.stride)
+    for sec, rows, nb, byte in (("gate_up_scales", 2 * F, H // 32, 0 if x_dtype == gw.BF16 else 103),
+                                ("down_scales", H, F // 32, 103)):
+        sc = r.integers(117, 123, size=(E, rows, nb), dtype=np.uint8)
+        np.put_along_axis(sc, r.integers(0, nb, size=(E, rows, 1)), np.uint8(byte), axis=2)
+        raw[:, layout.offsets[sec]:layout.offsets[sec] + rows * nb] = sc.reshape(E, -1)
+    buf.upload(raw)
+    xb, xw = _x(ctx, r, T, H, x_dtype)
+    logits = np.zeros((T, E), np.float32)
+    logits[np.arange(T), r.permutation(np.repeat(np.arange(E), counts))] = 4.0
+    lb = ctx.buffer(logits)
+    got = {}
+    for entries in ("0", "1000000"):
+        monkeypatch.setenv("GODWIT_WIDE_ENTRIES", entries)
+        runner = gw.ExpertRunner(ctx, H, F, act)
+        out, _, ids, _ = _run(ctx, runner, layout, buf, E, 1, xb, x_dtype, lb, T, H)
+        act_bits = _download(ctx, runner.prefill_view()["activations"], np.uint16, T * F)
+        got[entries] = out, act_bits, ids
+        runner.close()
+    for i in range(3):
+        assert np.array_equal(got["0"][i], got["1000000"][i]), i
+    y, off = _fp64_layer(layout, raw, got["0"][2][:, 0], xw.reshape(T, H), H, F, act)
+    err = np.abs(got["0"][0] - y)
+    assert np.all(err <= off), (err / off).max()
+    for b in (xb, lb, buf):
+        b.free()
