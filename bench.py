@@ -80,10 +80,10 @@ COUNTER_LAYERS = L
 #   gate_up_kernel, GPT-OSS-120B layer, batch 1 (profiles/decode_gate_up_down_traffic.md)
 GATE_UP_TRAFFIC = (35_944_526, "gw_kernels.hip", None)
 #   prefill gate_up GEMM, 512 tokens, seed 1 (profiles/prefill_gemm_gptoss_512.md)
-PREFILL_GATE_UP_TRAFFIC = (1_248_476_753, "gw_prefill.hip", "860aff5c4858a1d0")
+PREFILL_GATE_UP_TRAFFIC = (1_248_960_643, "gw_prefill.hip", "eed3117b8ed3141f")
 #   decode_layer_kernel (the one-kernel layer), GPT-OSS-120B, batch 1, over the
 #   whole 36-layer stack (profiles/decode_layer_traffic.md)
-DECODE_LAYER_TRAFFIC = (54_464_331, "gw_decode.hip", "257b3802b8b06735")
+DECODE_LAYER_TRAFFIC = (54_471_248, "gw_decode.hip", "e2752cd37aec17c7")
 
 
 def source_sha16(name: str) -> str:
